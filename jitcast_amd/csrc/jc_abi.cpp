@@ -149,8 +149,8 @@ LpKernel lp_choice(bool ts) {
     return ts ? kLpStream : kLpPersist;
 }
 
-// JITCAST_HIP_GEMM=own runs the plain GEMMs on the library's own MFMA kernels (gemm_f32, gemm_lp)
-// instead of hipBLASLt. Read at every call.
+// JITCAST_HIP_GEMM=own runs the plain GEMMs on the library's own MFMA kernels (gemm_f32_split,
+// gemm_lp) instead of hipBLASLt. Read at every call.
 bool use_blas(const jc_ctx* ctx) {
     if (!ctx->blas) return false;
     const char* e = getenv("JITCAST_HIP_GEMM");
@@ -883,16 +883,25 @@ static int launch_linear(jc_ctx* ctx, const char* W, const float* a, int lda, co
     if (bias) flags |= JC_GEMM_BIAS;
     int rc = check_linear(W, a, lda, w, bias, c, ldc, m, n, k, flags);
     if (rc || (size_t)m * n == 0) return rc;
-    if (use_blas(ctx)) {
+    const jc::GemmArgs g{a, w, bias, c, m, n, k, lda, ldc, flags};
+    const bool blas = use_blas(ctx), split = jc::gemm_f32_split_fits(g);
+    // hipBLASLt keeps the shapes too small to fill the chip with tiles (its 16- and 32-row tiles take
+    // 8 us and more; its fp32 rate is 100 to 145 TFLOP/s from there on): 333 x 768 x 3,072 19 us against
+    // 60, 148 x 512 x 512 8 against 13; 665 x 2,304 x 768 28 against 23, 2,660 x 768 x 768 31 against 27.
+    if (split && (!blas || jc::gemm_f32_split_us(g) < 8.f + 2.f * (float)m * (float)n * (float)k / 115e6f)) {
+        ProfScope ps(ctx, "gemm fp32 (fp16 pairs)");
+        const hipError_t e = jc::gemm_f32_split_launch(g, ctx->stream);
+        return e == hipSuccess ? JC_OK : hip_fail(W, e);
+    }
+    if (blas) {
         ProfScope ps(ctx, "gemm fp32 (hipBLASLt)");
         const jc::BlasStatus bs = jc::blas_gemm(ctx->blas, a, lda, w, bias, c, ldc, m, n, k, flags, JC_F32, JC_F32,
                                                 ctx->stream);
         if (bs == jc::kBlasDone) return JC_OK;
         if (bs == jc::kBlasError) return fail(JC_EHIP, "%s: hipblasLtMatmul failed", W);
     }
-    jc::GemmArgs g{a, w, bias, c, m, n, k, lda, ldc, flags};
-    ProfScope ps(ctx, "gemm_f32");
-    hipError_t e = jc::gemm_f32_launch(g, ctx->stream);
+    ProfScope ps(ctx, split ? "gemm fp32 (fp16 pairs)" : "gemm_f32");
+    const hipError_t e = split ? jc::gemm_f32_split_launch(g, ctx->stream) : jc::gemm_f32_launch(g, ctx->stream);
     return e == hipSuccess ? JC_OK : hip_fail(W, e);
 }
 

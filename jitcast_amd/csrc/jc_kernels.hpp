@@ -81,6 +81,11 @@ struct GemmArgs {
 };
 // k a multiple of 16; lda a multiple of 4; a, w 16-byte aligned
 hipError_t gemm_f32_launch(const GemmArgs& g, hipStream_t stream);
+// The same product on fp16 MFMA, each fp32 product as three fp16 ones (gemm_f32_split.hip); the same
+// conditions, and lda and k below 2^21 (gemm_f32_split_fits: a tile's rows span less than 2^31 bytes).
+bool gemm_f32_split_fits(const GemmArgs& g);
+float gemm_f32_split_us(const GemmArgs& g);  // its estimated time
+hipError_t gemm_f32_split_launch(const GemmArgs& g, hipStream_t stream);
 // y = x * (1 / sqrt(mean(x^2) + eps)) * w per row of d (d a multiple of 4; w may be null)
 hipError_t rms_norm_f32_launch(const float* x, float* y, const float* w, int rows, int d, float eps, hipStream_t stream);
 
