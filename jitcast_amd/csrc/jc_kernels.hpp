@@ -12,6 +12,8 @@ namespace jc {
 // Chronos-2 (ts = false) or Timestral (ts = true) time attention (time_mask.hpp); a.qgroups is set
 // by the launcher. fp32: dh a multiple of 8, at most 128; bf16/fp16: a multiple of 16, at most 128.
 hipError_t time_attention_f32_launch(const TimeArgs& a, int dh, bool ts, hipStream_t stream);
+// 64-wide heads, fp32 products on fp16 MFMA (time_attention_f32_split.hip)
+hipError_t time_attention_f32_split_launch(const TimeArgs& a, bool ts, hipStream_t stream);
 // Chronos-2 with 64-wide heads only (else hipErrorInvalidValue): out is fp16 [rows*n, 3*inner], each
 // output value's three-term split [hi | hi | lo] (the JC_F16X3 layer's A operand of the O projection).
 hipError_t time_attention_f32_x3_launch(const TimeArgs& a, int dh, hipStream_t stream);

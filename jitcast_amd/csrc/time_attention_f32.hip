@@ -691,6 +691,7 @@ static hipError_t dispatch_f32(const TimeArgs& a, int dh, hipStream_t stream) {
 
 hipError_t time_attention_f32_launch(const TimeArgs& a, int dh, bool ts, hipStream_t stream) {
     if (dh < 8 || dh > 128 || dh % 8) return hipErrorInvalidValue;
+    if (dh == 64) return time_attention_f32_split_launch(a, ts, stream);
     return ts ? dispatch_f32<true>(a, dh, stream) : dispatch_f32<false>(a, dh, stream);
 }
 
