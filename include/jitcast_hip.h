@@ -51,8 +51,7 @@ typedef struct jc_plan jc_plan;
 
 /* ---- runtime (replaces TornadoVM device selection and buffers: J/tornado/Devices.java:44-73) ---- */
 
-/* Makes `device` current and creates the context's stream (default priority) and its 64 KB buffer
- * for the group kernels' tile order (jc_c2_group_attention). */
+/* Makes `device` current and creates the context's stream (default priority). */
 int jc_init(int device, jc_ctx **ctx);
 /* Destroys the context (idempotent on NULL). */
 int jc_destroy(jc_ctx *ctx);
@@ -101,8 +100,6 @@ int jc_version(void);
  * jc_plan_launch, as the reference uploads them before each execution.
  */
 int jc_plan_begin(jc_ctx *ctx, uint64_t shape_key);
-/* (jc_plan_begin also allocates the plan's own 64 KB tile-order buffer, freed with the plan and not
- * counted by jc_plan_device_bytes.) */
 /* Ends the capture and instantiates the plan; on error no plan is made and capture has ended. */
 int jc_plan_end(jc_ctx *ctx, jc_plan **plan);
 /* Replays the plan on the context's current stream (asynchronous; jc_sync waits). */
@@ -181,8 +178,6 @@ int jc_c2_time_attention(jc_ctx *ctx, const void *qkv, void *out, const int32_t 
  * about 2^-20 of the fp32 product; a wave that meets a value beyond fp16's range runs on fp32 MFMA.
  * With JC_BF16 / JC_F16, K and Q enter the MFMA of their type as stored (exact products), and P as a
  * hi + lo pair of the type against V as stored.
- * A one-workgroup kernel first sorts the 16-row tiles by work (into the context's buffer, or the
- * plan's while capturing), so the launch dispatches the heaviest first.
  */
 int jc_c2_group_attention(jc_ctx *ctx, const void *qkv, void *out, const int32_t *live, const int32_t *group_start,
                           const int32_t *group_end, int rows, int n, int heads, int dh, int inner, int dtype);

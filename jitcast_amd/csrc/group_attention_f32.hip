@@ -22,14 +22,15 @@
 // The stage reads q|k|v once and writes out once, about 10 flop per byte: it is HBM-bound, so the
 // kernel is built around the memory stream. One wave per (16-row tile, slot) owns the groups that
 // START in its tile (found by a ballot on groupStart[i] == i), so each row's q, k and v are fetched
-// from HBM once; everything lives in registers (no LDS, no barriers). A one-workgroup kernel
-// (group_tile_order) first sorts the tiles by work, and the grid dispatches the heaviest first, so
-// the launch ends on light waves. The wave's work is a flat
+// from HBM once; everything lives in registers (no LDS, no barriers). Blocks run tile by tile, slots and
+// head ranges innermost, so consecutive blocks (one tile's, of like work) go to different XCDs. The
+// wave's work is a flat
 // stream of jobs (group, chunk of up to 4 query tiles (2 for heads over 64 wide), head, 16-key
 // tile): the chunk's queries and output accumulators stay in registers while the group's key tiles
 // stream past, each K/V tile used by every query tile right after it lands, and the next job's K/V loads are issued before this
 // job's MFMAs (register double-buffering). The online softmax across key tiles makes any group size
-// work; a group past 64 rows re-streams its keys once per further 64-row chunk.
+// work; a group past 64 rows re-streams its keys once per further 64-row chunk, which the wave of
+// the tile where that chunk's rows begin takes, so no wave holds a long group's queries alone.
 //
 // Operand layouts (16x16x4 f32: A lane i+16kk = A[i][kk], B lane j+16kk = B[kk][j]; 16x16x16
 // f16 / bf16: A lane i+16kk = A[i][4kk..4kk+3], B likewise by column; D lane j+16g reg r =
@@ -128,14 +129,13 @@ __global__ __launch_bounds__(kWave) void group_attention_f32(const GroupArgs a, 
     const int rows = a.rows, n = a.n, heads = a.heads, inner = a.inner;
     const int lane = threadIdx.x;
     const int j = lane % 16, g = lane / 16;
-    const uint32_t total = (uint32_t)a.rtiles * n * a.hsplit;
-    // With a tile order: blocks in that order (tile, then slot, then head range), heaviest first, so
-    // the last waves of the launch are light ones; consecutive blocks go to different XCDs, which
-    // balances them. Without: tiles fastest within each slot, each XCD a contiguous range.
-    const uint32_t logical = a.order ? blockIdx.x : xcd_remap(blockIdx.x, total);
+    // Tile by tile, in order, over the XCDs. (Sorting the tiles heaviest first by a kernel ahead of this
+    // one costs 5 us and gained nothing over it: 4,096 x 129, groups of 1..64, 1.225 against 1.232 ms;
+    // 1,300 x 133 in fives, bf16, 0.268 against 0.274. Slot by slot, each XCD a contiguous range: 1.337 and
+    // 0.278.)
+    const uint32_t logical = blockIdx.x;
     const uint32_t tile_slot = logical / a.hsplit;
-    const int t = a.order ? (int)(tile_slot % n) : (int)(tile_slot / a.rtiles);
-    const int rt = a.order ? a.order[tile_slot / n] : (int)(tile_slot % a.rtiles);
+    const int t = (int)(tile_slot % n), rt = (int)(tile_slot / n);
     // this wave's heads [h_lo, h_hi): a (tile, slot)'s heads are split over hsplit waves, so the
     // tiles where long groups start do not hold one wave for all heads while their neighbours idle
     const int hs = logical % a.hsplit;
@@ -147,10 +147,14 @@ __global__ __launch_bounds__(kWave) void group_attention_f32(const GroupArgs a, 
     const bool enc_slot = TS && t < a.enc;
     const bool cov = TS && a.covariates != 0 && a.role != nullptr;
 
-    // the groups starting in this tile (both bounds loaded at once: one round trip)
+    // the groups, and the further chunks of groups, starting in this tile (both bounds loaded at once: one
+    // round trip): the rows a whole number of chunks past their group's first
+    constexpr int kChunk = kRT * kQT;
     const int gs_l = lane < nr ? a.gstart[r0 + lane] : -1;
     const int ge_l = lane < nr ? a.gend[r0 + lane] : 0;
-    const uint32_t starts = (uint32_t)__ballot(gs_l == r0 + lane) & 0xffffu;
+    const int past = r0 + lane - gs_l;
+    const uint32_t starts =
+        (uint32_t)__ballot(gs_l >= 0 && past >= 0 && past % kChunk == 0 && (past == 0 || r0 + lane < ge_l)) & 0xffffu;
     if (starts == 0) return;
 
     // A tile of one-row groups (every series of the block univariate): a row's only key is itself,
@@ -202,12 +206,12 @@ __global__ __launch_bounds__(kWave) void group_attention_f32(const GroupArgs a, 
         Job jb;
         jb.valid = rest != 0;
         int b = jb.valid ? __builtin_ctz(rest) : 0;
-        jb.gs = r0 + b;
+        jb.gs = jb.valid ? __builtin_amdgcn_readlane(gs_l, b) : r0;
         // clamped into [gs+1, rows]: a group always holds its first row and only rows that exist.
         // Its end comes from the prologue's load (lane b holds gend[r0 + b]; b is wave-uniform), not
         // from memory: a load here would stall every group change on its latency.
         jb.ge = jb.valid ? min(max(__builtin_amdgcn_readlane(ge_l, b), jb.gs + 1), rows) : jb.gs + 1;
-        jb.qc = 0;
+        jb.qc = (r0 + b - jb.gs) / kChunk;
         jb.h = h_lo;
         jb.kt = 0;
         jb.pb = 1u;
@@ -231,8 +235,6 @@ __global__ __launch_bounds__(kWave) void group_attention_f32(const GroupArgs a, 
         if (++jb.kt < tiles) return jb;
         jb.kt = 0;
         if (++jb.h < h_hi) return jb;
-        jb.h = h_lo;
-        if (++jb.qc * kQT < tiles) return jb;
         return first_of(jb.rest);
     };
     // K (A operand) and V^T (A operand of PV) of a job's key tile; rows past the group are clamped
@@ -559,58 +561,11 @@ static int group_f32_mfma() {
     return e && e[0] == '1' ? 1 : 0;
 }
 
-constexpr int kOrderBuckets = 64;
-
-// A counting sort of the tiles by work into buckets, 0 for the most: a group's jobs per head are its
-// key tiles times its query tiles, (ceil(g / 16))^2 for a group of g rows (bounds clamped as the
-// kernel clamps them), summed over the groups starting in the tile. One row per lane (16 lanes a
-// tile, summed by shuffles), the buckets in LDS, one wave's scan of the counts, then the scatter.
-// Ties come out in any order: which block runs a tile changes nothing in its results.
-__global__ __launch_bounds__(1024) void group_tile_order(const int32_t* gstart, const int32_t* gend, int rows,
-                                                         int32_t* order) {
-    __shared__ int slot[kOrderBuckets];
-    __shared__ uint8_t bucket[kGroupOrderTiles];
-    const int tid = threadIdx.x, rtiles = (rows + kRT - 1) / kRT;
-    if (tid < kOrderBuckets) slot[tid] = 0;
-    __syncthreads();
-    for (int r = tid; r < rtiles * kRT; r += blockDim.x) {  // blockDim.x is a multiple of 16
-        int w = 0;
-        if (r < rows) {
-            const int gs = gstart[r], ge = gend[r];
-            if (gs == r) {
-                const int kt = min((min(max(ge, r + 1), rows) - r + kRT - 1) / kRT, kOrderBuckets);
-                w = kt * kt;
-            }
-        }
-#pragma unroll
-        for (int o = kRT / 2; o > 0; o >>= 1) w += __shfl_xor(w, o, kRT);
-        if (r % kRT == 0) {
-            const int b = kOrderBuckets - 1 - min(w, kOrderBuckets - 1);
-            bucket[r / kRT] = (uint8_t)b;
-            atomicAdd(&slot[b], 1);
-        }
-    }
-    __syncthreads();
-    if (tid < kOrderBuckets) {  // wave 0: exclusive prefix sum of the counts
-        const int c = slot[tid];
-        int x = c;
-#pragma unroll
-        for (int o = 1; o < kOrderBuckets; o <<= 1) {
-            const int y = __shfl_up(x, o);
-            if (tid >= o) x += y;
-        }
-        slot[tid] = x - c;
-    }
-    __syncthreads();
-    for (int tile = tid; tile < rtiles; tile += blockDim.x) order[atomicAdd(&slot[bucket[tile]], 1)] = tile;
-}
-
 template <typename T, int DHP, bool TS, bool EXACT, bool X3 = false>
 static hipError_t launch_group(GroupArgs a, int dh, hipStream_t stream) {
     a.rtiles = (a.rows + kRT - 1) / kRT;
     a.hsplit = std::min(group_head_split(), a.heads);
     a.f32_mfma = group_f32_mfma();
-    if (a.rtiles > kGroupOrderTiles) a.order = nullptr;
     const uint64_t grid = (uint64_t)a.rtiles * a.n * a.hsplit;
     if (grid > 0xffffffffull) return hipErrorInvalidValue;
     hipLaunchKernelGGL((group_attention_f32<T, DHP, TS, EXACT, X3>), dim3((uint32_t)grid), dim3(kWave), 0, stream, a,
@@ -646,13 +601,6 @@ hipError_t group_attention_launch(const GroupArgs& a, int dh, bool ts, int dtype
         case 2: return dispatch_group_type<_Float16>(a, dh, ts, stream);
         default: return hipErrorInvalidValue;
     }
-}
-
-hipError_t group_tile_order_launch(const int32_t* gstart, const int32_t* gend, int rows, int32_t* order,
-                                   hipStream_t stream) {
-    if (rows <= 0 || (rows + kRT - 1) / kRT > kGroupOrderTiles || !gstart || !gend || !order) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(group_tile_order, dim3(1), dim3(1024), 0, stream, gstart, gend, rows, order);
-    return hipGetLastError();
 }
 
 hipError_t group_attention_f32_x3_launch(const GroupArgs& a, int dh, hipStream_t stream) {
