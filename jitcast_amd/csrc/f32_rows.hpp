@@ -21,7 +21,7 @@ namespace jc {
 
 // Queries q0 + i (i < 16, below n) with bit i of `write` set are stored. words[b]: the validity word of
 // key block b (64 keys); trow(t): the RoPE table row of token t.
-template <bool ROPE, bool TS, typename Trow>
+template <bool ROPE, bool TS, bool X3, typename Trow>
 __device__ __forceinline__ void f32_rows(const TimeArgs& a, const TimeMask<TS>& mask, const uint64_t* words, Trow trow,
                                          int r, int h, int q0, uint32_t write, int lane) {
     constexpr int kDH = 64, kT = 16;
@@ -104,7 +104,12 @@ __device__ __forceinline__ void f32_rows(const TimeArgs& a, const TimeMask<TS>& 
 #pragma unroll
                 for (int u = 0; u < 4; u++) v[u] *= 1.f / (1.f + fast_exp2(-gv[u] * kLog2e));
             }
-            *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + at + 16 * t) = v;
+            if constexpr (X3) {  // [hi | hi | lo] rows, each value's three-term split
+                store_split_row(static_cast<_Float16*>(a.out) + ((size_t)r * n + q0 + i) * 3 * inner, inner,
+                                h * kDH + 4 * kk + 16 * t, v);
+            } else {
+                *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + at + 16 * t) = v;
+            }
         }
     }
 }

@@ -1,4 +1,5 @@
-// Time attention, fused flash-style for gfx950: the FP32 path of Chronos-2 and Timestral.
+// Time attention, fused flash-style for gfx950: the FP32 path of Chronos-2 and Timestral on fp32 MFMA, for the
+// head widths other than 64.
 //
 // Chronos-2 replaces the per-layer pair Chronos2Kernels.rope + Chronos2Kernels.timeAttention
 // (Chronos2Kernels.java:87-116, 118-464; oracle CpuChronos2.java:175-228, 284-304): unscaled scores
@@ -24,23 +25,7 @@
 // K/V/table prefetch uses buffer loads; keys past the end of the row fall outside the resource and
 // read as 0 (and are masked), so the load path has no per-lane bounds branches.
 //
-// FOLD (Chronos-2, rows of 128k + 1 tokens: [REG] after 128k patches): the row's last query would
-// be alone in a fifth workgroup that stages every K/V block for one query. The last full workgroup
-// computes it instead, on VALU beside its MFMA tiles: lane (key 8w + l/8, c = l%8) of wave w takes
-// dims 8c..8c+7 of one key of each 32-key block (8 products and an 8-lane DPP sum give the score),
-// each wave keeps a lazy online softmax over its 8 keys per block and accumulates its share of the
-// output from V^T in LDS, and the four shares are rescaled to a common max once at the end.
-//
-// The last key (Chronos-2, 64-wide heads, rows of 32k + 1 tokens): key n - 1 would be alone in a
-// last 32-key block whose MFMAs and staging cost a full block. It is staged once instead (rotated K
-// and V in LDS), and before the block loop each query takes its score against it on VALU (a 32-dim
-// dot per lane, summed over the lane pair) as the first step of its online softmax: running max
-// = that score, sum = 1, O = V[n - 1]. The folded query adds it in its final combination.
-//
-// X3 (Chronos-2, 64-wide heads; the JC_F16X3 layer): out is the O projection's A operand, fp16
-// rows of 3 * inner values [hi | hi | lo] (the three-term split of each fp32 output value), so the
-// layer needs no separate split pass over the attention output.
-#include "f32_tail.hpp"
+// Heads of exactly 64 run on time_attention_f32_split.hip.
 #include "jc_common.hpp"
 #include "jc_kernels.hpp"
 #include "time_mask.hpp"
@@ -63,14 +48,7 @@ struct F32Lds {
     float vt[2][kTiles * 32 * kPitchV];
     uint64_t mask[kMaxTokens / kMaskBlock];  // per 64-key word: key validity bits
     int32_t pos[TS ? kMaxTokens : 1];       // table row of every token of the row (Timestral)
-    float fold_q[DHP];                       // FOLD: the folded query, rotated and scaled
-    float last_k[DHP], last_v[DHP];          // the last key (rotated, unscaled) and its value
 };
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, (int)kRsrcWord3);
@@ -148,12 +126,10 @@ struct KvStage {
 };
 
 // EXACT: the head is exactly DHP wide, so every head-width expression folds to a constant
-template <int DHP, int KB, bool ROPE, bool TS, bool EXACT, bool FOLD, bool X3>
+template <int DHP, int KB, bool ROPE, bool TS, bool EXACT>
 __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a, int dh_rt) {
     const int dh = EXACT ? DHP : dh_rt;
-    static_assert(!X3 || (!TS && EXACT && DHP == 64), "split output: Chronos-2, 64-wide heads");
     static_assert(DHP % 16 == 0 && DHP <= 128, "head width");
-    static_assert(!FOLD || (!TS && EXACT && DHP == 64 && KB == 32), "the folded query: Chronos-2, 64-wide heads");
     static_assert(KB == 32 || KB == 64, "key block");
     constexpr int kHalfP = DHP / 2;
     constexpr int kSteps = kHalfP;  // K=2 per MFMA step: one dim from each lane half
@@ -167,39 +143,9 @@ __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a,
     const int n = a.n, inner = a.inner, half = dh / 2;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const int j = lane % 32, g = lane / 32;
-    const uint32_t items = (uint32_t)a.rows * a.heads;
-    // With tail workgroups (q_tail > 0), every 4 (row, head) items get their qgroups main
-    // workgroups followed by one tail workgroup whose 4 waves take the items' last R queries; the
-    // neighbouring logical workgroups run on one XCD, so the tail's K/V reads find them in its L2.
-    constexpr bool kTailOk = !TS && !FOLD && EXACT && DHP == 64 && KB == 32;  // FOLD rows have R = 1
-    const bool tails = kTailOk && a.q_tail > 0;
-    const uint32_t per_group = 4 * a.qgroups + 1;
-    const uint32_t total = tails ? (items + 3) / 4 * per_group : items * a.qgroups;
-    const uint32_t logical = xcd_remap(blockIdx.x, total);
-    int qg, bh;
-    if (tails) {
-        const uint32_t grp = logical / per_group, s = logical % per_group;
-        if (s == 4 * (uint32_t)a.qgroups) {
-            const uint32_t item = 4 * grp + tid / kWave;
-            if constexpr (kTailOk) {
-                if (item < items)
-                    f32_tail_item<ROPE, X3>(a, item / a.heads, item % a.heads, a.q_tail, tid % kWave);
-            }
-            return;  // the whole workgroup: tail workgroups take no barrier
-        }
-        const uint32_t item = 4 * grp + s / a.qgroups;
-        if (item >= items) return;  // the last group's missing items: before any barrier
-        qg = s % a.qgroups;
-        bh = item;
-    } else {
-        qg = logical % a.qgroups;
-        bh = logical / a.qgroups;
-    }
+    const uint32_t logical = xcd_remap(blockIdx.x, (uint32_t)a.rows * a.heads * a.qgroups);
+    const int qg = logical % a.qgroups, bh = logical / a.qgroups;
     const int h = bh % a.heads, r = bh / a.heads;
-    const bool fold = FOLD && qg == a.qgroups - 1;  // this workgroup also computes query n - 1
-    // key n - 1 alone in the last block: taken on VALU after the loop
-    constexpr bool kLastOk = !TS && EXACT && DHP == 64 && KB == 32;
-    const bool lastk = kLastOk && a.n > 1 && a.n % KB == 1;
     TimeMask<TS> mask;
     mask.init(a, r);
     const int32_t* vrow = a.valid + (size_t)r * (TS ? a.enc : n);
@@ -250,25 +196,11 @@ __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a,
         for (int t = tid; t < n; t += kThreads)
             lds.pos[t] = a.pos ? min(max(a.pos[(size_t)r * n + t], 0), a.table_rows - 1) : t;
     }
-    if (FOLD && fold && wave == 0 && lane < DHP / 2) {
-        // the folded query's dims e and e + 32, rotated at table row n - 1 like the tiles' queries
-        const int qf = n - 1, e = lane;
-        const float* qp = qkv + ((size_t)r * n + qf) * 3 * inner + h * dh;
-        float x = qp[e], y = qp[DHP / 2 + e];
-        if (ROPE) {
-            const float c = a.table[(size_t)qf * dh + e], sn = a.table[(size_t)qf * dh + DHP / 2 + e];
-            const float rx = x * c - y * sn, ry = y * c + x * sn;
-            x = rx;
-            y = ry;
-        }
-        lds.fold_q[e] = x * a.qscale;
-        lds.fold_q[DHP / 2 + e] = y * a.qscale;
-    }
     __syncthreads();
     // 64-key words any query of the workgroup can see (the same in every wave)
     const int qlo = qg * kWaves * kQ, qhi = min(qlo + kWaves * kQ, n) - 1;
     const uint64_t need = __ballot(lane < nwords && mask.any_allowed(lds.mask[lane], lane * kMaskBlock, qlo, qhi));
-    const int nblk = (n - (lastk ? 1 : 0) + KB - 1) / KB;
+    const int nblk = (n + KB - 1) / KB;
     auto next_block = [&](int after) {
         const int b = after + 1;
         const int w = b * KB / kMaskBlock;
@@ -313,58 +245,12 @@ __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a,
         stage.load(rk_at(kb), ROPE ? rt_at(kb) : rk_at(kb), lds.pos, kb * KB, n, tid, inner, dh);
         stage.store(lds, 0, tid);
     }
-    if (kLastOk && lastk && wave == 1) {
-        // key n - 1's dims e and e + 32, rotated at its table row as staging rotates every key (loaded
-        // here, after Q's prologue registers are free, beside the first block's staging)
-        const int kl = n - 1;
-        const float* kp = qkv + ((size_t)r * n + kl) * 3 * inner + inner + h * dh;
-        if (lane < DHP / 2) {
-            const int e = lane;
-            float x = kp[e], y = kp[DHP / 2 + e];
-            if (ROPE) {
-                const float c = a.table[(size_t)kl * dh + e], sn = a.table[(size_t)kl * dh + DHP / 2 + e];
-                const float rx = x * c - y * sn, ry = y * c + x * sn;
-                x = rx;
-                y = ry;
-            }
-            lds.last_k[e] = x;
-            lds.last_k[DHP / 2 + e] = y;
-        }
-        lds.last_v[lane] = kp[inner + lane];
-    }
     __syncthreads();
 
     floatx16 o_acc[kTiles];
 #pragma unroll
     for (int t = 0; t < kTiles; t++) o_acc[t] = floatx16{0};
     float m_run = -INFINITY, l_run = 0.f;
-    if (kLastOk && lastk && ((lds.mask[(n - 1) / kMaskBlock] >> ((n - 1) % kMaskBlock)) & 1ull)) {
-        // the live last key opens the online softmax (uniform over the workgroup): m = its score,
-        // P = 1, O = its value. Lane (j, g) holds dims 32g..32g+31 of query j, so the pair sum of
-        // the lane's partial dot is the whole score.
-        const float* kp = &lds.last_k[g * kHalfP];
-        float d = 0.f;
-#pragma unroll
-        for (int s4 = 0; s4 < kSteps / 4; s4++) {
-            const floatx4 kv = *reinterpret_cast<const floatx4*>(kp + 4 * s4);
-#pragma unroll
-            for (int u = 0; u < 4; u++) d += qreg[4 * s4 + u] * kv[u];
-        }
-        m_run = pair_sum(d);
-        l_run = g == 0 ? 1.f : 0.f;  // the pair sum at the end counts it once
-#pragma unroll
-        for (int t = 0; t < kTiles; t++) {
-#pragma unroll
-            for (int a4 = 0; a4 < 4; a4++) {
-                const floatx4 vv = *reinterpret_cast<const floatx4*>(&lds.last_v[32 * t + 8 * a4 + 4 * g]);
-#pragma unroll
-                for (int u = 0; u < 4; u++) o_acc[t][4 * a4 + u] = vv[u];
-            }
-        }
-    }
-    // FOLD: this wave's softmax state for the folded query over its keys (8 per block)
-    float f_m = -INFINITY, f_l = 0.f;
-    floatx4 f_oa = floatx4{0.f, 0.f, 0.f, 0.f}, f_ob = f_oa;
     int buf = 0;
     // Settle every prologue load here: the compiler cannot prove that the divergent Q loads were
     // consumed on all paths and would otherwise wait on them (vmcnt(0)) inside every iteration.
@@ -453,149 +339,14 @@ __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a,
                 }
             }
         }
-        if (FOLD && fold) {
-            // the folded query against key 8w + l/8 of the block: dims 8c..8c+7 in this lane
-            const int fkey = 8 * wave + lane / 8, c8 = 8 * (lane % 8);
-            const float* kr = &lds.k[buf][fkey * PK + c8];
-            const floatx4 ka = *reinterpret_cast<const floatx4*>(kr);
-            const floatx4 kb4 = *reinterpret_cast<const floatx4*>(kr + 4);
-            const floatx4 qa4 = *reinterpret_cast<const floatx4*>(&lds.fold_q[c8]);
-            const floatx4 qb4 = *reinterpret_cast<const floatx4*>(&lds.fold_q[c8 + 4]);
-            float sc = 0.f;
-#pragma unroll
-            for (int u = 0; u < 4; u++) sc += ka[u] * qa4[u] + kb4[u] * qb4[u];
-            sc += dpp_f<0xB1>(sc);   // quad_perm [1,0,3,2]
-            sc += dpp_f<0x4E>(sc);   // quad_perm [2,3,0,1]
-            sc += dpp_f<0x141>(sc);  // row_half_mirror: the key's 8 lanes hold its score
-            const bool live = (word >> ((k0 % kMaskBlock) + fkey)) & 1ull;
-            const float fs = live ? sc : -INFINITY;
-            // the reference max moves only when a score passes it by 2^64 (or at the first live key),
-            // so P stays below 2^64
-            if (__any(fs - f_m > 64.f)) {
-                float mx = fmaxf(fs, dpp_f<0x128>(fs));  // row_ror:8: the row's other key
-                auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-                mx = pair_max(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])));
-                const float m_new = fmaxf(f_m, mx);
-                const float alpha = fast_exp2(f_m - m_new);  // f_m = -inf: 0
-                f_l *= alpha;
-                f_oa *= alpha;
-                f_ob *= alpha;
-                f_m = m_new;
-            }
-            const float p = live ? fast_exp2(fs - f_m) : 0.f;
-            f_l += p;
-            const float* vp = &lds.vt[buf][c8 * PV + fkey];  // V[key][c8 + u] at row c8 + u of V^T
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                f_oa[u] += p * vp[u * PV];
-                f_ob[u] += p * vp[(4 + u) * PV];
-            }
-        }
         if (next < nblk) stage.store(lds, buf ^ 1, tid);
         __syncthreads();
         buf ^= 1;
         kb = next;
     }
 
-    if (FOLD && fold) {
-        // each wave's share: dims 8c..8c+7 summed over its 8 keys' lanes (c, c+8, ..., c+56), with its
-        // max and sum (each key's P counted in 8 lanes), into the K buffers (free after the loop)
-        floatx4 fo[2] = {f_oa, f_ob};
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                float v = fo[i][u];
-                v += dpp_f<0x128>(v);  // row_ror:8
-                auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-                fo[i][u] = pair_sum(__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
-            }
-        }
-        float lw = f_l;
-        lw += dpp_f<0xB1>(lw);
-        lw += dpp_f<0x4E>(lw);
-        lw += dpp_f<0x124>(lw);  // row_ror:4
-        lw += dpp_f<0x128>(lw);  // row_ror:8
-        {
-            auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(lw), __float_as_uint(lw), false, false);
-            lw = pair_sum(__uint_as_float(sw[0]) + __uint_as_float(sw[1])) * 0.125f;
-        }
-        float* part = &lds.k[0][wave * (DHP + 2)];
-        if (lane < 8) {
-            *reinterpret_cast<floatx4*>(&part[8 * lane]) = fo[0];
-            *reinterpret_cast<floatx4*>(&part[8 * lane + 4]) = fo[1];
-        }
-        if (lane == 0) {
-            part[DHP] = f_m;
-            part[DHP + 1] = lw;
-        }
-        __syncthreads();
-        if (wave == 0) {
-            float mw[kWaves], mx = -INFINITY;
-#pragma unroll
-            for (int w = 0; w < kWaves; w++) {
-                mw[w] = lds.k[0][w * (DHP + 2) + DHP];
-                mx = fmaxf(mx, mw[w]);
-            }
-            // the folded query against the last key, when the loop left it out and it is live
-            float sl = -INFINITY;
-            if (lastk && ((lds.mask[(n - 1) / kMaskBlock] >> ((n - 1) % kMaskBlock)) & 1ull)) {
-                float d = lds.fold_q[lane] * lds.last_k[lane];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off);
-                sl = d;
-                mx = fmaxf(mx, sl);
-            }
-            float o = 0.f, l = 0.f;
-            if (mx != -INFINITY) {
-#pragma unroll
-                for (int w = 0; w < kWaves; w++) {
-                    const float f = fast_exp2(mw[w] - mx);
-                    o += f * lds.k[0][w * (DHP + 2) + lane];
-                    l += f * lds.k[0][w * (DHP + 2) + DHP + 1];
-                }
-                const float f = fast_exp2(sl - mx);  // 0 without the last key
-                o += f * lds.last_v[lane];
-                l += f;
-            }
-            const float res = l > 0.f ? o / l : 0.f;
-            if constexpr (X3) {
-                store_split_one(static_cast<_Float16*>(a.out) + ((size_t)r * n + n - 1) * 3 * inner, inner,
-                                h * dh + lane, res);
-            } else {
-                float* op = static_cast<float*>(a.out) + ((size_t)r * n + n - 1) * inner + h * dh;
-                op[lane] = res;
-            }
-        }
-    }
-
     // every lane reaches the swap (its partner holds the other half of the same query)
     const float l = pair_sum(l_run);
-    if constexpr (X3) {
-        // Lanes (j, 0) and (j, 1) trade halves of each 16-dim run (v_permlane32_swap), so each holds 8
-        // consecutive dims: 32t + 16p + 8g + (0..7), from O^T regs 8p + u (dims 32t + 16p + 4g + u) and
-        // 8p + 4 + u (dims 32t + 16p + 8 + 4g + u). Each piece of the split then goes out as one
-        // 16-byte store.
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        _Float16* orow = static_cast<_Float16*>(a.out) + ((size_t)r * n + q0 + j) * 3 * inner + h * dh;
-#pragma unroll
-        for (int t = 0; t < kTiles; t++) {
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                floatx4 d0, d4;
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(o_acc[t][8 * p + u] * inv),
-                                                                     __float_as_uint(o_acc[t][8 * p + 4 + u] * inv),
-                                                                     false, false);
-                    d0[u] = __uint_as_float(sw[0]);
-                    d4[u] = __uint_as_float(sw[1]);
-                }
-                if (j < nq) store_split_row8(orow, inner, 32 * t + 16 * p + 8 * g, d0, d4);
-            }
-        }
-        return;
-    }
     if (j < nq) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
         const size_t tok = (size_t)r * n + q0 + j;
@@ -626,52 +377,13 @@ __global__ __launch_bounds__(kThreads) void time_attention_f32(const TimeArgs a,
 
 }  // namespace
 
-template <int DHP, int KB, bool TS, bool EXACT, bool FOLD, bool X3>
-static void launch_f32_rope(const TimeArgs& a, int dh, uint64_t grid, hipStream_t stream) {
-    if (a.table) {
-        hipLaunchKernelGGL((time_attention_f32<DHP, KB, true, TS, EXACT, FOLD, X3>), dim3((uint32_t)grid),
-                           dim3(kThreads), 0, stream, a, dh);
-    } else {
-        hipLaunchKernelGGL((time_attention_f32<DHP, KB, false, TS, EXACT, FOLD, X3>), dim3((uint32_t)grid),
-                           dim3(kThreads), 0, stream, a, dh);
-    }
-}
-
-// R when a row of 128k + R tokens, 2 <= R <= 16, takes tail workgroups for its last R queries
-// (Chronos-2, 64-wide heads, no gate), else 0
-static int tail_rows(const TimeArgs& a, int dh) {
-    if (dh != 64 || a.gate || a.q_begin != 0 || a.n <= kWaves * kQ) return 0;
-    if (a.table && a.table_rows < a.n) return 0;
-    const int R = a.n % (kWaves * kQ);
-    return R >= 2 && R <= kTailT ? R : 0;
-}
-
-template <int DHP, bool TS, bool EXACT, bool X3 = false>
+template <int DHP, bool TS, bool EXACT>
 static hipError_t launch_f32(TimeArgs a, int dh, hipStream_t stream) {
-    constexpr int KB = 32;  // 32-key blocks (64 measured slower on config 1)
-    const int tiles = (a.n + kQ - 1) / kQ;
-    // a last query alone after whole workgroups (n = 128k + 1) is folded into the last of them
-    constexpr bool kCanFold = !TS && EXACT && DHP == 64;
-    const bool fold = kCanFold && a.n > 1 && a.n % (kWaves * kQ) == 1;
-    a.qgroups = fold ? (a.n - 1) / (kWaves * kQ) : (tiles + kWaves - 1) / kWaves;
-    // rows of 128k + R tokens, 2 <= R <= 16 (Chronos-2, 64-wide heads): the main workgroups take the
-    // first 128k queries and tail workgroups (f32_tail.hpp) the last R, instead of a fifth main
-    // workgroup that stages every block for one partly filled wave
-    int tail = 0;
-    if constexpr (kCanFold) tail = tail_rows(a, dh);
-    if (tail) {
-        a.qgroups = (a.n - tail) / (kWaves * kQ);
-        a.q_tail = a.n - tail;
-    }
-    const uint64_t items = (uint64_t)a.rows * a.heads;
-    const uint64_t grid = tail ? (items + 3) / 4 * (4 * a.qgroups + 1) : items * a.qgroups;
-    if constexpr (kCanFold) {
-        if (fold) {
-            launch_f32_rope<DHP, KB, TS, EXACT, true, X3>(a, dh, grid, stream);
-            return hipGetLastError();
-        }
-    }
-    launch_f32_rope<DHP, KB, TS, EXACT, false, X3>(a, dh, grid, stream);
+    constexpr int KB = 32;  // 32-key blocks (64 measured slower at 256 x 513 tokens)
+    a.qgroups = (a.n + kWaves * kQ - 1) / (kWaves * kQ);
+    const dim3 grid((uint32_t)((uint64_t)a.rows * a.heads * a.qgroups)), block(kThreads);
+    if (a.table) hipLaunchKernelGGL((time_attention_f32<DHP, KB, true, TS, EXACT>), grid, block, 0, stream, a, dh);
+    else hipLaunchKernelGGL((time_attention_f32<DHP, KB, false, TS, EXACT>), grid, block, 0, stream, a, dh);
     return hipGetLastError();
 }
 
@@ -684,7 +396,7 @@ template <bool TS>
 static hipError_t dispatch_f32(const TimeArgs& a, int dh, hipStream_t stream) {
     if (dh <= 16) return launch_f32_width<16, TS>(a, dh, stream);
     if (dh <= 32) return launch_f32_width<32, TS>(a, dh, stream);
-    if (dh <= 64 || !TS) return launch_f32_width<64, TS>(a, dh, stream);
+    if (dh <= 64) return launch_f32<64, TS, false>(a, dh, stream);
     if constexpr (TS) return launch_f32_width<128, TS>(a, dh, stream);  // Chronos-2 heads are at most 64 wide
     return hipErrorInvalidValue;
 }
@@ -693,11 +405,6 @@ hipError_t time_attention_f32_launch(const TimeArgs& a, int dh, bool ts, hipStre
     if (dh < 8 || dh > 128 || dh % 8) return hipErrorInvalidValue;
     if (dh == 64) return time_attention_f32_split_launch(a, ts, stream);
     return ts ? dispatch_f32<true>(a, dh, stream) : dispatch_f32<false>(a, dh, stream);
-}
-
-hipError_t time_attention_f32_x3_launch(const TimeArgs& a, int dh, hipStream_t stream) {
-    if (dh != 64) return hipErrorInvalidValue;
-    return launch_f32<64, false, true, true>(a, dh, stream);
 }
 
 int time_attention_max_tokens() { return kMaxTokens; }

@@ -5,6 +5,8 @@ import pytest
 import torch
 
 from jitcast_amd import chronos2, timestral
+from tests.test_gpu_stage import _run_layer
+from tests.test_oracle_ops import _layer_weights
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -136,3 +138,23 @@ def test_timestral(gpu, enc, h, gate, factor):
     for r in range(rows):
         for hh in range(heads):
             assert _err(out[r, :, hh], exp[r, :, hh]) <= TOL
+
+
+@pytest.mark.parametrize("n,quiet", [(37, 0), (129, 0), (37, 32), (133, 33), (260, 40)])
+def test_split_output(gpu, n, quiet):
+    """The split rows that the f16x3 layer's O projection reads, against the fp32 layer. The `quiet` first tokens
+    are so small that the scales they set overflow at the others: those queries come from the recomputation."""
+    print(f"case f16x3 layer n={n} quiet={quiet}", flush=True)
+    rows, heads, d, dff = 3, 2, 64, 128
+    r = np.random.default_rng(n + quiet)
+    w = _layer_weights(n, d, heads * DH, dff, False)
+    x = r.standard_normal((rows, n, d)).astype(np.float32)
+    x[:, :quiet] *= 1e-9  # rms norm's eps leaves them at 1e-6 of the others
+    live = np.ones((rows, n), np.int32)
+    live[1, : n // 4] = 0
+    group = np.array([0, 0, 1], np.int32)
+    out = [_run_layer(x.reshape(-1, d), w, live, group, rows, n, heads, DH, dff, 1e-6, t).astype(np.float64)
+           for t in ("f16x3", None)]
+    assert np.isfinite(out[0]).all()
+    # three terms of fp16 pairs leave 2^-22 of a product, and at most 2^-25 absolute of a value below fp16's range
+    assert np.linalg.norm(out[0] - out[1]) <= 1e-5 * np.linalg.norm(out[1])
