@@ -126,20 +126,20 @@ void prof_clear(jc_ctx* ctx) {
     ctx->prof->clear();
 }
 
-// JITCAST_HIP_LP_KERNEL picks the bf16/fp16 time-attention kernel: "stream" (time_attention_lp,
-// which takes every shape), "wide" (time_attention_lpw) or "persist" (time_attention_lpp), the
-// last two for the shapes they take ("persist" covers time_attention_lpp, rows of 257..513 tokens,
-// and time_attention_lps, rows of 65..160). Unset, Chronos-2 uses a persistent kernel where one
-// fits, else the row-wide one, and Timestral the streaming one: its row-wide variant holds every token's
-// table row in LDS and fits one workgroup per CU (measured on config 3: 6.30 ms against 6.04 ms
-// per 12 layers). Read at every launch, so a host can switch at run time.
-enum LpKernel { kLpStream, kLpWide, kLpPersist };
-LpKernel lp_choice(bool ts) {
+// JITCAST_HIP_LP_KERNEL picks the bf16/fp16 time-attention kernel: "stream" (time_attention_lp, which takes
+// every shape), "wide" (time_attention_lpw for 32-wide heads and rows of 256 tokens or more, time_attention_lpr for
+// 64-wide ones and rows of 33 or more) or "persist" (Chronos-2's time_attention_lpp for rows of 257..513 tokens and
+// time_attention_lps for rows of 65..160, else as "wide"). Unset: a persistent kernel where it is worth it
+// (time_attention_lpp_worth, time_attention_lps_worth), else the ring kernel (time_attention_lpr), else Chronos-2's
+// row-wide and Timestral's streaming one (a row-wide workgroup that holds every token's table row fits once per CU).
+// Read at every launch, so a host can switch at run time.
+enum LpKernel { kLpAuto, kLpStream, kLpWide, kLpPersist };
+LpKernel lp_choice() {
     const char* e = getenv("JITCAST_HIP_LP_KERNEL");
     if (e && !strcmp(e, "stream")) return kLpStream;
     if (e && !strcmp(e, "wide")) return kLpWide;
     if (e && !strcmp(e, "persist")) return kLpPersist;
-    return ts ? kLpStream : kLpPersist;
+    return kLpAuto;
 }
 
 // JITCAST_HIP_GEMM=own runs the plain GEMMs on the library's own MFMA kernels (gemm_f32_split,
@@ -460,24 +460,29 @@ static int check_time_common(const char* W, const void* qkv, const void* out, co
     return JC_OK;
 }
 
-// fp32 goes to the fp32 kernel; bf16/fp16 to the row-wide kernel when lp_use_wide() picks it and
-// the shape fits it, else to the streaming kernel, which takes every shape. Both give the same
+// fp32 goes to the fp32 kernels; bf16/fp16 to the kernel lp_choice() picks where it fits the shape. All give the same
 // results to within rounding.
 static int launch_time(jc_ctx* ctx, const char* W, const jc::TimeArgs& a, int dh, bool ts, int dtype) {
     hipError_t e;
     const bool fp16 = dtype == JC_F16;
+    const LpKernel choice = lp_choice();
     if (dtype == JC_F32) {
         ProfScope ps(ctx, ts ? "ts time_attention_f32" : "c2 time_attention_f32");
         e = jc::time_attention_f32_launch(a, dh, ts, ctx->stream);
-    } else if (lp_choice(ts) == kLpPersist && jc::time_attention_lpp_fits(a, dh, ts)) {
-        ProfScope ps(ctx, ts ? "ts time_attention_lpp" : "c2 time_attention_lpp");
+    } else if (jc::time_attention_lpp_fits(a, dh, ts) &&
+               (choice == kLpPersist || (choice == kLpAuto && jc::time_attention_lpp_worth(a, ctx->cus)))) {
+        ProfScope ps(ctx, "c2 time_attention_lpp");
         e = jc::time_attention_lpp_launch(a, fp16, ctx->cus, ctx->stream);
-    } else if (lp_choice(ts) == kLpPersist && jc::time_attention_lps_fits(a, dh, ts)) {
-        ProfScope ps(ctx, ts ? "ts time_attention_lps" : "c2 time_attention_lps");
+    } else if (jc::time_attention_lps_fits(a, dh, ts) &&
+               (choice == kLpPersist || (choice == kLpAuto && jc::time_attention_lps_worth(a, ctx->cus)))) {
+        ProfScope ps(ctx, "c2 time_attention_lps");
         e = jc::time_attention_lps_launch(a, fp16, ctx->cus, ctx->stream);
-    } else if (lp_choice(ts) != kLpStream && jc::time_attention_lpw_fits(a, dh)) {
+    } else if (choice != kLpStream && jc::time_attention_lpr_fits(a, dh)) {
+        ProfScope ps(ctx, ts ? "ts time_attention_lpr" : "c2 time_attention_lpr");
+        e = jc::time_attention_lpr_launch(a, ts, fp16, ctx->stream);
+    } else if (choice != kLpStream && (!ts || choice != kLpAuto) && jc::time_attention_lpw_fits(a, dh)) {
         ProfScope ps(ctx, ts ? "ts time_attention_lpw" : "c2 time_attention_lpw");
-        e = jc::time_attention_lpw_launch(a, dh, ts, fp16, ctx->stream);
+        e = jc::time_attention_lpw_launch(a, ts, fp16, ctx->stream);
     } else {
         ProfScope ps(ctx, ts ? "ts time_attention_lp" : "c2 time_attention_lp");
         e = jc::time_attention_lp_launch(a, dh, ts, fp16, ctx->stream);

@@ -19,16 +19,23 @@ hipError_t time_attention_f32_split_launch(const TimeArgs& a, bool ts, hipStream
 hipError_t time_attention_f32_x3_launch(const TimeArgs& a, int dh, hipStream_t stream);
 hipError_t time_attention_lp_launch(const TimeArgs& a, int dh, bool ts, bool fp16, hipStream_t stream);
 int time_attention_max_tokens();
-// The row-wide bf16/fp16 kernel: 8-wave workgroups of 256 queries of one (row, head); dh 32 or 64;
-// rows of at least 256 tokens.
+// The row-wide bf16/fp16 kernel of 32-wide heads: 8-wave workgroups of 256 queries of one (row, head); rows of
+// at least 256 tokens.
 bool time_attention_lpw_fits(const TimeArgs& a, int dh);
-hipError_t time_attention_lpw_launch(const TimeArgs& a, int dh, bool ts, bool fp16, hipStream_t stream);
-// The persistent bf16/fp16 kernel (Chronos-2, dh 64, 257..513 tokens per row, no gate): one
-// 8-wave workgroup per CU streams its (row, head) items; `cus` sizes the grid.
+hipError_t time_attention_lpw_launch(const TimeArgs& a, bool ts, bool fp16, hipStream_t stream);
+// The persistent bf16/fp16 kernel of long rows (Chronos-2, dh 64, 257..513 tokens, no gate): one 8-wave workgroup
+// per CU streams its (row, head) items; `cus` sizes the grid. worth: whether it is faster there than the ring kernel.
 bool time_attention_lpp_fits(const TimeArgs& a, int dh, bool ts);
+bool time_attention_lpp_worth(const TimeArgs& a, int cus);
 hipError_t time_attention_lpp_launch(const TimeArgs& a, bool fp16, int cus, hipStream_t stream);
+// The persistent bf16/fp16 kernel of short rows (Chronos-2, dh 64, 65..160 tokens, no gate); `cus` sizes the grid.
+// worth: whether it is faster there than the ring kernel.
 bool time_attention_lps_fits(const TimeArgs& a, int dh, bool ts);
+bool time_attention_lps_worth(const TimeArgs& a, int cus);
 hipError_t time_attention_lps_launch(const TimeArgs& a, bool fp16, int cus, hipStream_t stream);
+// The ring kernel of bf16/fp16 rows of 33 tokens or more, dh 64 (time_attention_lpr.hip)
+bool time_attention_lpr_fits(const TimeArgs& a, int dh);
+hipError_t time_attention_lpr_launch(const TimeArgs& a, bool ts, bool fp16, hipStream_t stream);
 // att[i] *= sigmoid(g[i]) for i < count (dtype: 0 fp32, 1 bf16, 2 fp16)
 hipError_t gate_launch(void* att, const void* g, uint64_t count, int dtype, hipStream_t stream);
 // The arguments of the group-attention kernels (by value).

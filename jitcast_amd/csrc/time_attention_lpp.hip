@@ -584,6 +584,14 @@ bool time_attention_lpp_fits(const TimeArgs& a, int dh, bool ts) {
     return true;
 }
 
+// Its workgroups cover 512 queries and take the row's last one along: at 513 tokens 256 rows run 0.382 ms against
+// 0.434 on the ring kernel (time_attention_lpr.hip), 20 rows 0.045 against 0.056. Shorter rows leave query tiles
+// empty (250 x 300 0.247 against 0.214, 200 x 449 0.292 against 0.262, 256 x 512 0.388 against 0.378), and with few
+// items most CUs have none (4 x 513 0.035 against 0.022).
+bool time_attention_lpp_worth(const TimeArgs& a, int cus) {
+    return a.n > kPart && 4ull * a.rows * a.heads >= 3ull * cus;
+}
+
 hipError_t time_attention_lpp_launch(const TimeArgs& a, bool fp16, int cus, hipStream_t stream) {
     const uint64_t items = (uint64_t)a.rows * a.heads;
     if (items == 0) return hipSuccess;

@@ -423,6 +423,14 @@ bool time_attention_lps_fits(const TimeArgs& a, int dh, bool ts) {
     return true;
 }
 
+// Measured against the ring kernel (time_attention_lpr.hip), 12 heads: 1,000 rows of 133 tokens 0.248 against 0.32 ms,
+// 500 of 129 0.124 against 0.142, 260 of 133 0.072 against 0.070 alone but 1% of a layer ahead, 170 of 133 0.0506
+// against 0.0502; 900 of 128 0.180 against 0.193, but 1,000 of 96 0.186 against 0.176. With few items most CUs have
+// none (20 rows of 133: 0.109 against 0.010).
+bool time_attention_lps_worth(const TimeArgs& a, int cus) {
+    return a.n > 112 && (uint64_t)a.rows * a.heads >= 8ull * cus;
+}
+
 hipError_t time_attention_lps_launch(const TimeArgs& a, bool fp16, int cus, hipStream_t stream) {
     const uint64_t items = (uint64_t)a.rows * a.heads;
     if (items == 0) return hipSuccess;

@@ -1,4 +1,4 @@
-// Time attention for gfx950, bf16 / fp16: the row-wide kernel. One 8-wave workgroup covers 256
+// Time attention for gfx950, bf16 / fp16: the row-wide kernel of 32-wide heads. One 8-wave workgroup covers 256
 // queries (8 tiles of 32) of one (row, head), so each K/V block is loaded, rotated and transposed
 // once per 256 queries; two workgroups share a CU and run out of phase.
 //
@@ -482,19 +482,15 @@ hipError_t launch_lpw(TimeArgs a, hipStream_t stream) {
 }  // namespace
 
 bool time_attention_lpw_fits(const TimeArgs& a, int dh) {
-    if (dh != 32 && dh != 64) return false;
+    if (dh != 32) return false;  // 64-wide heads: time_attention_lpr.hip
     if (a.n < 256) return false;  // 8 tiles or more: short rows keep the streaming kernel
     if (a.table && (a.table_rows + kKB - 1) / kKB > kMaxHi) return false;
     return true;
 }
 
-hipError_t time_attention_lpw_launch(const TimeArgs& a, int dh, bool ts, bool fp16, hipStream_t stream) {
-    if (fp16) {
-        if (dh == 32) return ts ? launch_lpw<_Float16, 32, true>(a, stream) : launch_lpw<_Float16, 32, false>(a, stream);
-        return ts ? launch_lpw<_Float16, 64, true>(a, stream) : launch_lpw<_Float16, 64, false>(a, stream);
-    }
-    if (dh == 32) return ts ? launch_lpw<__bf16, 32, true>(a, stream) : launch_lpw<__bf16, 32, false>(a, stream);
-    return ts ? launch_lpw<__bf16, 64, true>(a, stream) : launch_lpw<__bf16, 64, false>(a, stream);
+hipError_t time_attention_lpw_launch(const TimeArgs& a, bool ts, bool fp16, hipStream_t stream) {
+    if (fp16) return ts ? launch_lpw<_Float16, 32, true>(a, stream) : launch_lpw<_Float16, 32, false>(a, stream);
+    return ts ? launch_lpw<__bf16, 32, true>(a, stream) : launch_lpw<__bf16, 32, false>(a, stream);
 }
 
 }  // namespace jc
