@@ -394,8 +394,9 @@ int64_t jc_c2_layer_workspace_bytes(int rows, int n, int d, int inner, int dff, 
  * accumulation (the reference's FP16 GEMM modes, Chronos2Forward.java:377-409, GemmMode.HALF), both
  * attention cores read q|k|v and write their output in the storage type (fp32 arithmetic inside),
  * and x (the residual stream), the norms and the accumulations stay fp32. JC_F16X3 (no reference counterpart): every
- * GEMM runs on its operands' three-term fp16 splits (jc_split_f16x3; the norms, and the attention
- * kernels for 64-wide heads, write the split directly), with fp32 accumulation and fp32 outputs;
+ * GEMM runs on its operands' three-term fp16 splits with fp32 accumulation and fp32 outputs. The weights come
+ * as jc_split_f16x3 rows. Large GEMMs split their fp32 activations themselves, each row scaled first, so none is out
+ * of range; for the others the kernel before them writes the split (saturated to +-65504, as jc_split_f16x3);
  * the attention, the norms and x are fp32, as in JC_F32, whose accuracy it keeps to about 2^-20 per
  * product (plus 2^-25 times the other operand where lo is subnormal, for operands below about
  * 2^-2).

@@ -29,6 +29,11 @@
 // 2,304 x 768 0.381 ms (hipBLASLt 0.985), 768 x 768 0.147 (0.363), 3,072 x 768 0.505 (1.262), 768 x
 // 3,072 0.477 (1.212). Error against 64 bits (2-norm, N(0, 1) times N(0, 0.02)): 3.2e-7 at k = 768, 6.2e-7
 // at k = 3,072; fp32 MFMA 5.0e-7 and 7.0e-7 to 9.9e-7 (a k-step adds 16 products before it rounds).
+//
+// W as split rows (JC_F16X3 layers: pairs made once by jc_split_f16x3, unscaled) skips W's half of the conversion:
+// a layer of 34,580 rows whose GEMMs all run so 2.40 ms, with fp32 W 2.45.
+#include <type_traits>
+
 #include "jc_common.hpp"
 #include "jc_kernels.hpp"
 #include "lp_common.hpp"
@@ -134,7 +139,46 @@ struct Operand {
     }
 };
 
-template <int BM, int BN, int WM, int WN>
+// W's rows as jc_split_f16x3 wrote them ([hi | lo | hi], 3k fp16 values; the third part is not read): the pairs
+// pass to the stage as they are, with no scale. The interface is Operand's.
+template <int NI, int STEP>
+struct SplitOperand {
+    halfx8 hi[NI], lo[NI];
+
+    __device__ __forceinline__ void init() {}
+    __device__ __forceinline__ void load(const _Float16* p, int rows, uint32_t row_bytes, uint32_t tid, int st, int stages, int k) {
+        const uint32_t half = (st == stages - 1 && (k & 16)) ? kOutOfRange : 0u;
+        const uint32_t t = tid;
+        const uint32_t o = ((t / 4) * row_bytes + 16u * (t % 4)) | (t << 30 & half);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int left = st < stages ? rows - i * STEP : 0;
+            const uint32_t bytes = left > 0 ? (uint32_t)(left - 1) * row_bytes + (uint32_t)(k - st * kSK) * 2u : 0u;
+            const char* base = reinterpret_cast<const char*>(p) + (size_t)i * STEP * row_bytes + (size_t)st * kSK * 2;
+            hi[i] = __builtin_bit_cast(halfx8, __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(base, bytes), o, 0, 0));
+            lo[i] = __builtin_bit_cast(halfx8, __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(base + (size_t)k * 2, bytes), o, 0, 0));
+        }
+    }
+    __device__ __forceinline__ void set_scales() {}
+    template <int N>
+    __device__ __forceinline__ void store(uint16_t (&part)[2][N], uint32_t tid, int i0 = 0, int i1 = NI) {
+        const uint32_t t = tid;
+#pragma unroll
+        for (int i = i0; i < i1; i++) {
+            const uint32_t o = sswz(t / 4, t % 4) + i * STEP * kSK;
+            *reinterpret_cast<halfx8*>(&part[0][o]) = hi[i];
+            *reinterpret_cast<halfx8*>(&part[1][o]) = lo[i];
+        }
+    }
+    __device__ __forceinline__ void finish(int32_t* e, uint32_t tid) const {
+        if (tid % 4) return;
+#pragma unroll
+        for (int i = 0; i < NI; i++) e[tid / 4 + i * STEP] = 0;
+    }
+};
+
+// XW: g.w holds split rows (SplitOperand) instead of fp32 ones.
+template <bool XW, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_f32_split(const GemmArgs g, uint32_t tiles_n, uint32_t total,
                                                                     int vec) {
     constexpr int kThreads = WM * WN * kWave;
@@ -152,13 +196,16 @@ __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_f32_split(const GemmA
     const int m0 = (int)(tile / tiles_n) * BM, n0 = (int)(tile % tiles_n) * BN;
     const int stages = (g.k + kSK - 1) / kSK;
 
-    const float *pa = g.a + (size_t)m0 * g.lda, *pw = g.w + (size_t)n0 * g.k;
+    using WT = std::conditional_t<XW, _Float16, float>;
+    const size_t ldw = (XW ? 3 : 1) * (size_t)g.k;  // a row of W, in its own elements
+    const float* pa = g.a + (size_t)m0 * g.lda;
+    const WT* pw = reinterpret_cast<const WT*>(g.w) + (size_t)n0 * ldw;
     const int rows_a = min(BM, g.m - m0), rows_w = min(BN, g.n - n0);
     Operand<NA, kStep> oa;
-    Operand<NW, kStep> ow;
+    std::conditional_t<XW, SplitOperand<NW, kStep>, Operand<NW, kStep>> ow;
     oa.init();
     ow.init();
-    const uint32_t a_row = (uint32_t)g.lda * 4u, w_row = (uint32_t)g.k * 4u;
+    const uint32_t a_row = (uint32_t)g.lda * 4u, w_row = (uint32_t)(ldw * sizeof(WT));
     oa.load(pa, rows_a, a_row, tid, 0, stages, g.k);
     ow.load(pw, rows_w, w_row, tid, 0, stages, g.k);
     floatx16 acc[TM][TN];
@@ -271,11 +318,17 @@ __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_f32_split(const GemmA
                 // on fp32 MFMA from the operands themselves: lane (i, hg) contracts k = 8q + 4hg + u
                 // with step u
                 const float* ta = g.a + (size_t)min(m0 + rb + j, g.m - 1) * g.lda + 4 * hg;
-                const float* tw = g.w + (size_t)min(n0 + cb + j, g.n - 1) * g.k + 4 * hg;
+                const WT* tw = reinterpret_cast<const WT*>(g.w) + (size_t)min(n0 + cb + j, g.n - 1) * ldw + 4 * hg;
                 floatx16 t = floatx16{0};
                 for (int q = 0; q < g.k; q += 8) {
                     const floatx4 av = *reinterpret_cast<const floatx4*>(ta + q);
-                    const floatx4 wv = *reinterpret_cast<const floatx4*>(tw + q);
+                    floatx4 wv;
+                    if constexpr (XW) {
+#pragma unroll
+                        for (int u = 0; u < 4; u++) wv[u] = (float)tw[q + u] + (float)tw[g.k + q + u];
+                    } else {
+                        wv = *reinterpret_cast<const floatx4*>(tw + q);
+                    }
 #pragma unroll
                     for (int u = 0; u < 4; u++) t = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], wv[u], t, 0, 0, 0);
                 }
@@ -342,12 +395,12 @@ __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_f32_split(const GemmA
     }
 }
 
-template <int BM, int BN, int WM, int WN>
+template <bool XW, int BM, int BN, int WM, int WN>
 hipError_t launch_split(const GemmArgs& g, hipStream_t stream) {
     const uint32_t tn = (uint32_t)((g.n + BN - 1) / BN);
     const uint64_t total = (uint64_t)((g.m + BM - 1) / BM) * tn;
     const int vec = g.ldc % 4 == 0 && (size_t)g.c % 16 == 0;
-    hipLaunchKernelGGL((gemm_f32_split<BM, BN, WM, WN>), dim3((uint32_t)total), dim3(WM * WN * kWave), 0, stream, g, tn,
+    hipLaunchKernelGGL((gemm_f32_split<XW, BM, BN, WM, WN>), dim3((uint32_t)total), dim3(WM * WN * kWave), 0, stream, g, tn,
                        (uint32_t)total, vec);
     return hipGetLastError();
 }
@@ -376,18 +429,25 @@ int best_tiling(const GemmArgs& g) {
     return best;
 }
 
+template <bool XW>
+hipError_t launch_best(const GemmArgs& g, hipStream_t stream) {
+    switch (best_tiling(g)) {
+        case 0: return launch_split<XW, 256, 256, 2, 4>(g, stream);
+        case 1: return launch_split<XW, 128, 128, 2, 2>(g, stream);
+        default: return launch_split<XW, 64, 64, 2, 2>(g, stream);
+    }
+}
+
 }  // namespace
 
 bool gemm_f32_split_fits(const GemmArgs& g) { return g.lda < (1 << 21) && g.k < (1 << 21); }
 
+bool gemm_f32_split_w_fits(const GemmArgs& g) { return g.lda < (1 << 21) && g.k < (1 << 20); }
+
 float gemm_f32_split_us(const GemmArgs& g) { return tiling_us(g, best_tiling(g)); }
 
-hipError_t gemm_f32_split_launch(const GemmArgs& g, hipStream_t stream) {
-    switch (best_tiling(g)) {
-        case 0: return launch_split<256, 256, 2, 4>(g, stream);
-        case 1: return launch_split<128, 128, 2, 2>(g, stream);
-        default: return launch_split<64, 64, 2, 2>(g, stream);
-    }
-}
+hipError_t gemm_f32_split_launch(const GemmArgs& g, hipStream_t stream) { return launch_best<false>(g, stream); }
+
+hipError_t gemm_f32_split_w_launch(const GemmArgs& g, hipStream_t stream) { return launch_best<true>(g, stream); }
 
 }  // namespace jc

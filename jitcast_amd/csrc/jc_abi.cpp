@@ -1123,10 +1123,34 @@ int jc_split_f16x3(jc_ctx* ctx, const float* src, int ld_src, void* dst, int row
     return launch_split_x3(ctx, W, src, ld_src, dst, rows, k, weights);
 }
 
-// The JC_F32 layer with every GEMM on the operands' three-term fp16 splits: the norms write the
-// A-operand split of hn directly, the attention kernels write the split of their outputs (64-wide
-// heads; other widths go through fp32 and a split pass), the MLP activation is split before its
-// GEMM, and every GEMM (K = 3k, fp32 accumulation) writes fp32.
+// Whether a JC_F16X3 layer's GEMM takes its A operand in fp32 (gemm_f32_split.hip splits it on the way to LDS) and
+// not as a split that the kernel before it wrote, `extra` bytes a value more than fp32 (2 from a norm or an attention
+// kernel, 10 from a pass). Both run at about 1 PFLOP/s of fp16 products; hipBLASLt's smaller tiles fill the last
+// round better. 768 wide, 34,580 rows, the layer: all GEMMs on splits 2.57 ms, the down projection on fp32 A 2.42,
+// all 2.40; 13,167 rows 0.966, 0.969, 1.072; 5,320 rows 0.437, 0.448, 0.497; 333 rows 0.122, 0.151, 0.172.
+static bool x3_plain_a(jc_ctx* ctx, int m, int n, int k, int extra) {
+    const jc::GemmArgs g{nullptr, nullptr, nullptr, nullptr, m, n, k, k, n, 0};
+    if (!jc::gemm_f32_split_w_fits(g)) return false;
+    if (!use_blas(ctx)) return true;
+    return jc::gemm_f32_split_us(g) < 6.f * (float)m * (float)n * (float)k / 1e9f + (float)extra * (float)m * (float)k / 5.2e6f;
+}
+
+// One GEMM of a JC_F16X3 layer: a is fp32 [m, k] (plain) or its A-operand split [m, 3k], w the W-operand split.
+static int x3_linear(jc_ctx* ctx, const char* W, const void* a, bool plain, const void* w, const float* bias, float* c,
+                     int m, int n, int k, int flags) {
+    if (!plain) return launch_linear_lp(ctx, W, a, 3 * k, w, bias, c, n, m, n, 3 * k, flags, JC_F16, JC_F32);
+    if (bias) flags |= JC_GEMM_BIAS;
+    if (!aligned16(w)) return fail(JC_EINVAL, "%s: a and w must be 16-byte aligned", W);
+    ProfScope ps(ctx, "gemm f16x3 (fp16 pairs)");
+    const jc::GemmArgs g{static_cast<const float*>(a), static_cast<const float*>(w), bias, c, m, n, k, k, n, flags};
+    const hipError_t e = jc::gemm_f32_split_w_launch(g, ctx->stream);
+    return e == hipSuccess ? JC_OK : hip_fail(W, e);
+}
+
+// The JC_F32 layer with every GEMM on fp16 pairs, its weights split once by the caller. Where x3_plain_a says so a
+// GEMM splits its A operand itself; else it is an fp16 GEMM over K = 3k with the A-operand split written by the
+// kernel before it (the norm, the attention kernel for 64-wide heads) or by a pass (other widths, the MLP
+// activation). All accumulate and write fp32.
 static int layer_x3(jc_ctx* ctx, const char* W, float* x, const jc_c2_layer_weights* w, const int32_t* live,
                     const float* table, const int32_t* group_start, const int32_t* group_end, void* workspace, int rows,
                     int n, int d, int heads, int dh, int dff, float eps) {
@@ -1136,51 +1160,38 @@ static int layer_x3(jc_ctx* ctx, const char* W, float* x, const jc_c2_layer_weig
     char* ws = static_cast<char*>(workspace);
     float* big = reinterpret_cast<float*>(ws);                                  // qkv [T, 3*inner] or act [T, dff]
     float* att = reinterpret_cast<float*>(ws + round256(t * big_cols * 4));    // [T, inner]
-    void* a3 = ws + round256(t * big_cols * 4) + round256(t * (size_t)inner * 4);  // [T, 3k] fp16, k <= max(d, inner, dff)
-    const int F = JC_F16;
+    void* a3 = ws + round256(t * big_cols * 4) + round256(t * (size_t)inner * 4);  // [T, 3k] fp16, k <= max(d, inner, dff), or the norm's [T, d] fp32
+    const bool pq = x3_plain_a(ctx, T, 3 * inner, d, 2), po = x3_plain_a(ctx, T, d, inner, dh == 64 ? 2 : 10);
+    const bool pu = x3_plain_a(ctx, T, dff, d, 2), pd = x3_plain_a(ctx, T, d, dff, 10);
     int rc;
-    auto rms3 = [&](const float* nw) -> int {
-        ProfScope ps(ctx, "rms_norm (split out)");
-        hipError_t e = jc::rms_norm_x3_launch(x, a3, nw, T, d, eps, ctx->stream);
+    auto rms = [&](const float* nw, bool plain) -> int {
+        ProfScope ps(ctx, plain ? "rms_norm_f32" : "rms_norm (split out)");
+        hipError_t e = plain ? jc::rms_norm_f32_launch(x, static_cast<float*>(a3), nw, T, d, eps, ctx->stream)
+                             : jc::rms_norm_x3_launch(x, a3, nw, T, d, eps, ctx->stream);
         return e == hipSuccess ? JC_OK : hip_fail(W, e);
     };
+    const bool fused = dh == 64 && !po;  // the attention kernels write the split themselves
+    const bool split = dh != 64 && !po;
+    const void* ao = po ? (const void*)att : a3;
     // time attention sub-layer (Chronos2Forward.java:260-271)
-    if ((rc = rms3(w->time_norm))) return rc;
-    if ((rc = launch_linear_lp(ctx, W, a3, 3 * d, w->time_qkv, w->time_qkv_bias, big, 3 * inner, T, 3 * inner, 3 * d, 0,
-                               F, JC_F32)))
-        return rc;
-    const bool fused = dh == 64;  // the attention kernels write the split themselves
-    if (fused) {
-        if ((rc = c2_time(ctx, W, big, a3, live, table, rows, n, heads, dh, inner, JC_F32, true))) return rc;
-    } else {
-        if ((rc = c2_time(ctx, W, big, att, live, table, rows, n, heads, dh, inner, JC_F32, false))) return rc;
-        if ((rc = launch_split_x3(ctx, W, att, inner, a3, T, inner, 0))) return rc;
-    }
-    if ((rc = launch_linear_lp(ctx, W, a3, 3 * inner, w->time_o, w->time_o_bias, x, d, T, d, 3 * inner,
-                               JC_GEMM_ACCUMULATE, F, JC_F32)))
-        return rc;
+    if ((rc = rms(w->time_norm, pq))) return rc;
+    if ((rc = x3_linear(ctx, W, a3, pq, w->time_qkv, w->time_qkv_bias, big, T, 3 * inner, d, 0))) return rc;
+    if ((rc = c2_time(ctx, W, big, fused ? a3 : att, live, table, rows, n, heads, dh, inner, JC_F32, fused))) return rc;
+    if (split && (rc = launch_split_x3(ctx, W, att, inner, a3, T, inner, 0))) return rc;
+    if ((rc = x3_linear(ctx, W, ao, po, w->time_o, w->time_o_bias, x, T, d, inner, JC_GEMM_ACCUMULATE))) return rc;
     // group attention sub-layer (Chronos2Forward.java:273-281)
-    if ((rc = rms3(w->group_norm))) return rc;
-    if ((rc = launch_linear_lp(ctx, W, a3, 3 * d, w->group_qkv, w->group_qkv_bias, big, 3 * inner, T, 3 * inner, 3 * d,
-                               0, F, JC_F32)))
+    if ((rc = rms(w->group_norm, pq))) return rc;
+    if ((rc = x3_linear(ctx, W, a3, pq, w->group_qkv, w->group_qkv_bias, big, T, 3 * inner, d, 0))) return rc;
+    if ((rc = c2_group(ctx, W, big, fused ? a3 : att, live, group_start, group_end, rows, n, heads, dh, inner, JC_F32,
+                       fused)))
         return rc;
-    if (fused) {
-        if ((rc = c2_group(ctx, W, big, a3, live, group_start, group_end, rows, n, heads, dh, inner, JC_F32, true)))
-            return rc;
-    } else {
-        if ((rc = c2_group(ctx, W, big, att, live, group_start, group_end, rows, n, heads, dh, inner, JC_F32, false)))
-            return rc;
-        if ((rc = launch_split_x3(ctx, W, att, inner, a3, T, inner, 0))) return rc;
-    }
-    if ((rc = launch_linear_lp(ctx, W, a3, 3 * inner, w->group_o, w->group_o_bias, x, d, T, d, 3 * inner,
-                               JC_GEMM_ACCUMULATE, F, JC_F32)))
-        return rc;
+    if (split && (rc = launch_split_x3(ctx, W, att, inner, a3, T, inner, 0))) return rc;
+    if ((rc = x3_linear(ctx, W, ao, po, w->group_o, w->group_o_bias, x, T, d, inner, JC_GEMM_ACCUMULATE))) return rc;
     // feed-forward sub-layer (Chronos2Forward.java:283-286)
-    if ((rc = rms3(w->mlp_norm))) return rc;
-    if ((rc = launch_linear_lp(ctx, W, a3, 3 * d, w->wi, w->wi_bias, big, dff, T, dff, 3 * d, JC_GEMM_RELU, F, JC_F32)))
-        return rc;
-    if ((rc = launch_split_x3(ctx, W, big, dff, a3, T, dff, 0))) return rc;
-    return launch_linear_lp(ctx, W, a3, 3 * dff, w->wo, w->wo_bias, x, d, T, d, 3 * dff, JC_GEMM_ACCUMULATE, F, JC_F32);
+    if ((rc = rms(w->mlp_norm, pu))) return rc;
+    if ((rc = x3_linear(ctx, W, a3, pu, w->wi, w->wi_bias, big, T, dff, d, JC_GEMM_RELU))) return rc;
+    if (!pd && (rc = launch_split_x3(ctx, W, big, dff, a3, T, dff, 0))) return rc;
+    return x3_linear(ctx, W, pd ? (const void*)big : a3, pd, w->wo, w->wo_bias, x, T, d, dff, JC_GEMM_ACCUMULATE);
 }
 
 // ---- The rest of the Chronos-2 forward ------------------------------------------------------

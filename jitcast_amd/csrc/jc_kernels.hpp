@@ -85,6 +85,9 @@ hipError_t gemm_f32_launch(const GemmArgs& g, hipStream_t stream);
 bool gemm_f32_split_fits(const GemmArgs& g);
 float gemm_f32_split_us(const GemmArgs& g);  // its estimated time
 hipError_t gemm_f32_split_launch(const GemmArgs& g, hipStream_t stream);
+// The same with w as fp16 [n, 3k], jc_split_f16x3's W rows, 16-byte aligned; k below 2^20.
+bool gemm_f32_split_w_fits(const GemmArgs& g);
+hipError_t gemm_f32_split_w_launch(const GemmArgs& g, hipStream_t stream);
 // y = x * (1 / sqrt(mean(x^2) + eps)) * w per row of d (d a multiple of 4; w may be null)
 hipError_t rms_norm_f32_launch(const float* x, float* y, const float* w, int rows, int d, float eps, hipStream_t stream);
 
