@@ -22,7 +22,8 @@
 // What bounds it: the latency of a block's step (4 waves per SIMD; at Timestral's 64 x 1,025 tokens, gate on, VALU 43% and
 // MFMA 18% of the cycles, LDS 21%). There 0.298 ms, 0.408 on the streaming kernel, whose workgroups of 128 queries staged
 // every block through registers (fp16 0.300 against 0.463); with its last part of one query as any other part 0.323.
-// Chronos-2: 90 x 197 0.039 (0.056), 383 x 245 0.170 (0.258), 64 x 577 0.128 (0.158 on the row-wide kernel). 5 .. 7 waves ran slower than 8 with idle ones (units of 8 keys then fall unevenly: 64 x
+// Chronos-2: 90 x 197 0.039 (0.056), 383 x 245 0.170 (0.258), 64 x 577 0.128 (0.158 on the row-wide kernel).
+// 5 .. 7 waves ran slower than 8 with idle ones (units of 8 keys then fall unevenly: 64 x
 // 1,025 on 7 waves 0.389); requesting the first blocks ahead of the validity scan cost short rows 8%.
 #include "jc_common.hpp"
 #include "jc_kernels.hpp"
